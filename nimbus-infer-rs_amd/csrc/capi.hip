@@ -171,9 +171,10 @@ nis::RowArgs row_args(const float* d_logits, int64_t ld, int64_t V, const nis_pa
 //   - other rows with V > 53245, no top-k: the 512-lane long-row kernel
 //     (greedy, top-p off or top-p, the row read again from cache after its
 //     stream), then the general path on the rows it declined;
-//   - anything else (V < 256, top-p <= 0, top-k with a penalty history or
-//     past 53245, a penalty history on rows longer than the registers hold):
-//     the 512-lane general kernel.
+//   - 0 < top-k < V with a penalty history, or with V > 53245 (to 262141), at
+//     any top-p > 0: the 1024-lane top-k path (only the row's head is kept);
+//   - anything else (V < 256, top-p <= 0, top-k past 262141, a penalty history
+//     on rows longer than the registers hold): the 512-lane general kernel.
 // A row one of these kernels cannot prove (non-finite values, capacity,
 // exact-tie overflow, a history past the bitmaps) runs the general path
 // inside whichever kernel was launched.
@@ -240,8 +241,17 @@ int launch_rows(nis_ctx* ctx, const nis::RowArgs& a, int32_t B) {
         // exact-tie overflow, a top-p row's span)
         hipLaunchKernelGGL(nis::sample_rows_pending_kernel, dim3((unsigned)std::min(B, 256)),
                            dim3(nis::kBlock), 0, ctx->stream, a, B);
+    } else if (nis::topk_eligible(a)) {
+        // top-k with a penalty history or on long rows: the smallest group
+        // that covers the row (16 groups per lane; V + 3 <= 65536 G)
+        if (a.V <= 65533)
+            hipLaunchKernelGGL(nis::sample_rows_kernel<1>, dim3((unsigned)B), dim3(nis::kTB), 0, ctx->stream, a);
+        else if (a.V <= 131069)
+            hipLaunchKernelGGL(nis::sample_rows_kernel<2>, dim3((unsigned)B), dim3(nis::kTB), 0, ctx->stream, a);
+        else
+            hipLaunchKernelGGL(nis::sample_rows_kernel<4>, dim3((unsigned)B), dim3(nis::kTB), 0, ctx->stream, a);
     } else {
-        hipLaunchKernelGGL(nis::sample_rows_kernel, dim3((unsigned)B), dim3(nis::kBlock), 0,
+        hipLaunchKernelGGL(nis::sample_rows_kernel<0>, dim3((unsigned)B), dim3(nis::kBlock), 0,
                            ctx->stream, a);
     }
     hipError_t e = hipGetLastError();

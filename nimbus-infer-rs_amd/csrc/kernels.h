@@ -5,18 +5,34 @@
 #include "dense_path.h"
 #include "long_path.h"
 #include "long_sparse_path.h"
+#include "topk_path.h"
 
 namespace nis {
 
-// One 512-lane workgroup per row on the general path: the launches no
-// row kernel takes (V < 256, top-p <= 0, top-k with a penalty history or on
-// rows longer than the registers hold, a penalty history on rows longer
-// than the registers hold).
-__global__ __launch_bounds__(kBlock) void sample_rows_kernel(RowArgs a) {
-    __shared__ GeneralShared sh;
+// The launches no other kernel takes.  G = 0: one 512-lane workgroup per row
+// on the general path (V < 256, top-p <= 0, a penalty history on rows longer
+// than the registers hold).  G = 1, 2, 4: one 1024-lane workgroup per row on
+// the top-k path, G float4s per group (top-k with a penalty history, or on
+// rows longer than the registers hold); a row it declines runs the general
+// path on the first 512 lanes, the other waves leaving first.
+template <int G>
+__global__ __launch_bounds__(G == 0 ? kBlock : kTB) void sample_rows_kernel(RowArgs a) {
     const int row = (int)blockIdx.x;
     if (a.done != nullptr && a.done[row]) return;  // a finished sequence (decode step)
-    general_row(a, row, sh, NIS_REJECT_SHAPE);
+    if constexpr (G == 0) {
+        __shared__ GeneralShared sh;
+        general_row(a, row, sh, NIS_REJECT_SHAPE);
+    } else {
+        __shared__ union {
+            GeneralShared g;
+            TopkShared t;
+        } sh;
+        const uint32_t reject = topk_row<G>(a, row, sh.t);
+        if (reject == NIS_REJECT_NONE) return;
+        if (threadIdx.x >= kBlock) return;
+        __syncthreads();
+        general_row<1>(a, row, sh.g, reject);
+    }
 }
 
 // Sparse top-p rows: one 1024-lane workgroup per row.  A row the sparse
