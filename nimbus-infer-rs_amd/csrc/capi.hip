@@ -15,6 +15,7 @@
 #include "kernels.h"
 #include "floor_path.h"
 #include "lm_head.h"
+#include "lm_head_split.h"
 
 // 16-row hidden tiles per matrix-core wave when B > 16 (4 or 2)
 #ifndef NIS_LH_NB
@@ -318,6 +319,43 @@ bool launch_lm_head_row(const nis::LmHeadArgs& a, bool grouped, uintptr_t wp, hi
     return true;
 }
 
+// The split-bf16 kernel (lm_head_split.h): 32, 64, 128 or 256 hidden rows per
+// workgroup by B, and the widest vocab tile that still gives at least 192 of
+// the 256 CUs a workgroup (x is split once per workgroup): 512 rows, 256, or
+// 128 in workgroups of 4 waves.
+template <int FMT, int NB, int NV, int NW>
+void launch_lm_head_split_n(const nis::LmHeadArgs& a, hipStream_t st) {
+    // (64 h a chunk; 32 where x's parts or f32 weights would take too much room)
+    constexpr int KT = FMT == nis::kLhF32 || (NB == 8 && FMT == nis::kLhInt8) ? 2 : 4;
+    const dim3 grid((unsigned)((a.V + 32 * NV * NW - 1) / (32 * NV * NW)), (unsigned)((a.B + 32 * NB - 1) / (32 * NB)));
+    hipLaunchKernelGGL((nis::lm_head_split_kernel<FMT, NB, NV, KT, NW>), grid, dim3(64 * NW), 0, st, a);
+}
+template <int FMT, int NB>
+void launch_lm_head_split_b(const nis::LmHeadArgs& a, hipStream_t st) {
+    if constexpr (NB <= 2)  // (4 x 2 tiles spill registers)
+        if (a.V >= 192 * 512) return launch_lm_head_split_n<FMT, NB, 2, 8>(a, st);
+    if (a.V >= 192 * 256) launch_lm_head_split_n<FMT, NB, 1, 8>(a, st);
+    else launch_lm_head_split_n<FMT, NB, 1, 4>(a, st);
+}
+template <int FMT>
+void launch_lm_head_split_f(const nis::LmHeadArgs& a, hipStream_t st) {
+    if (a.B <= 32) launch_lm_head_split_b<FMT, 1>(a, st);
+    else if (a.B <= 64) launch_lm_head_split_b<FMT, 2>(a, st);
+    else if (a.B <= 128 || FMT == nis::kLhInt4) launch_lm_head_split_b<FMT, 4>(a, st);
+    else launch_lm_head_split_b<FMT, FMT == nis::kLhInt4 ? 4 : 8>(a, st);
+}
+// Rows of W start on 4 bytes and no load crosses H (H % 4, for codes H % 8); a
+// group is whole MFMA steps of 32.
+// Returns false to leave the call to the f32 matrix-core kernel.
+bool launch_lm_head_split(const nis::LmHeadArgs& a, int fmt, bool grouped, uintptr_t wp, hipStream_t st) {
+    if (a.H > nis::kLsMaxH || a.ldx > (1 << 20) || (wp & 3u) != 0 || a.H % (fmt == NIS_W_F32 ? 4 : 8) != 0) return false;
+    if (grouped && a.group % 32 != 0) return false;
+    if (fmt == NIS_W_F32) launch_lm_head_split_f<nis::kLhF32>(a, st);
+    else if (fmt == NIS_W_INT8) launch_lm_head_split_f<nis::kLhInt8>(a, st);
+    else launch_lm_head_split_f<nis::kLhInt4>(a, st);
+    return true;
+}
+
 // Argument checks of the LM-head entry points, and their kernel arguments.
 int lm_head_setup(nis_ctx* ctx, const float* d_hidden, int64_t ldh, int32_t B, int32_t H,
                   const nis_weights* w, int64_t V, float* d_logits, int64_t ld, bool logits_optional,
@@ -545,6 +583,7 @@ int nis_lm_head_logits(nis_ctx* ctx, const float* d_hidden, int64_t ldh, int32_t
     } else if (B == 1) {
         if (launch_lm_head_row<nis::kLhInt4>(a, grouped, wp, ctx->stream)) goto launched;
     }
+    if (launch_lm_head_split(a, fmt, grouped, wp, ctx->stream)) goto launched;
     {
     // a wave: 64 vocab rows x 16*nb hidden rows; workgroups of 1 wave for
     // small batches (spread over every CU), else 4 waves split along b first
