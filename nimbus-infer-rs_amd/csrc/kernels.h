@@ -10,8 +10,8 @@
 namespace nis {
 
 // The launches no other kernel takes.  G = 0: one 512-lane workgroup per row
-// on the general path (V < 256, top-p <= 0, a penalty history on rows longer
-// than the registers hold).  G = 1, 2, 4: one 1024-lane workgroup per row on
+// on the general path (V < 256, top-p <= 0, a penalty history on top-p rows of
+// V > 262080).  G = 1, 2, 4: one 1024-lane workgroup per row on
 // the top-k path, G float4s per group (top-k with a penalty history, or on
 // rows longer than the registers hold); a row it declines runs the general
 // path on the first 512 lanes, the other waves leaving first.

@@ -25,9 +25,14 @@
 // float4s (few kept) or its chunks read a third time (few removed) ->
 // lanes -> elements.
 //
+// With a repetition-penalty history: see each mode (greedy and top-p off take
+// the penalised values in the stream, top-p from a list beside it).
+//
 // A row this path cannot prove returns a reject code before anything is
 // written, and the caller runs the general path on it.
 #pragma once
+#include <type_traits>
+
 #include "dense_path.h"
 
 namespace nis {
@@ -41,8 +46,9 @@ constexpr int kLQ = 64 * kLSpan / kLB;  // searched buckets per lane
 constexpr uint32_t kLPending = 0xFFF00000u;  // token of a declined row (| reject code)
 constexpr int kLMem = 2048;           // members of the cutoff bucket listed by the second read
 
-enum { kLongTopP = 0, kLongAll = 1, kLongGreedy = 2 };
-constexpr int kLPenMaxV = kLRing * 64 - 64;  // greedy with a penalty history: the bitmap's reach
+enum { kLongTopP = 0, kLongAll = 1, kLongGreedy = 2, kLongTopPPen = 3 };
+constexpr int kLPenMaxV = kLRing * 64 - 64;  // with a penalty history: the bitmap's reach
+constexpr int kLPen = 2048;                  // top-p: distinct penalised ids
 
 // A member of the cutoff bucket, listed by the second read.
 struct LMem {
@@ -71,6 +77,16 @@ struct LongShared {
     uint32_t cnt;                     // members of the final bucket
 };
 
+// Top-p with a penalty history, as well: the penalised ids and their values.
+struct LongPenShared : LongShared {
+    uint32_t bits[2 * kLRing];        // bit 4 s + q: element q of float4 slot s is penalised
+    double py[kLPen];                 // the distinct ones: value after the penalty,
+    uint32_t pid[kLPen];              //   row index
+    double my[kDMem];                 // the final bucket's penalised members' values
+    uint32_t np;
+};
+static_assert(sizeof(LongPenShared) <= 163840, "LDS of one workgroup");
+
 template <int MODE>
 __device__ __forceinline__ bool long_eligible(const RowArgs a, int row) {
     if (a.V < 256 || a.V > NIS_MAX_V) return false;
@@ -82,7 +98,8 @@ __device__ __forceinline__ bool long_eligible(const RowArgs a, int row) {
     }
     int64_t g0 = 0, g1 = 0;
     if (a.penalty != 1.0f && gen_range(a, row, g0, g1) && g1 > g0) {
-        // greedy and top-p off take the history as a bitmap over the ring's words
+        // greedy and top-p off take the history as a bitmap over the ring's
+        // words, kLongTopPPen as one of its own
         if (MODE == kLongTopP || a.V > kLPenMaxV) return false;
     }
     return true;
@@ -101,9 +118,11 @@ __device__ __forceinline__ bool long_eligible(const RowArgs a, int row) {
 constexpr uint32_t kLSpanRetry = 0x200u;  // (internal: never reported)
 constexpr uint32_t kLSpanFlag = 0x40000u; // pending token: retry with rfloor in the low 14 bits (+8192)
 template <int MODE>
-__device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, LongShared& sh,
+__device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
+                                             std::conditional_t<MODE == kLongTopPPen, LongPenShared, LongShared>& sh,
                                              uint32_t prior = NIS_REJECT_NONE, const float rfloor = -INFINITY,
                                              float* const rnext = nullptr) {
+    constexpr bool PP = MODE == kLongTopPPen, TOPP = MODE == kLongTopP || PP;
     const int l = lane_id();
     const int w = __builtin_amdgcn_readfirstlane(wave_id());
     const int tid = (int)threadIdx.x;
@@ -138,23 +157,45 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
     const float t0 = bcast_f32(hv, 3), t1 = bcast_f32(hv, 4), t2 = bcast_f32(hv, 5);
     const f4v ninf4 = f4v{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
     // the row's values of chunk k (outside the row: -inf)
-    auto fixc = [&](f4v v, int k) -> f4v {
+    auto fixr = [&](f4v v, int k) -> f4v {
         if (k >= Kw) return ninf4;
         const int fb0 = wbase + 64 * k;
         if (fb0 < f_lo || fb0 + 63 > f_hi)
             return fix_slot(v, slot0 + 64 * k, f_lo, f_hi, mis, V, h0, h1, h2, t0, t1, t2);
         return v;
     };
+    // PP: which elements of the lane's slot in chunk k < Kw are penalised
+    // (their float positions id + mis have a nibble per slot)
+    auto ppnib = [&](int k) -> uint32_t {
+        if constexpr (PP) {
+            const uint32_t s = (uint32_t)(slot0 + 64 * k);
+            return (sh.bits[s >> 3] >> (4u * (s & 7u))) & 15u;
+        }
+        return 0u;
+    };
+    // PP: the penalised elements are -inf here; each_pen adds their values
+    auto fixc = [&](f4v v, int k) -> f4v {
+        v = fixr(v, k);
+        if constexpr (PP)
+            if (k < Kw) v = d_mask4(v, ppnib(k));
+        return v;
+    };
 
     f4v buf[kLD];
     buf[0] = ld(0);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (MODE == kLongTopP) {
+    if constexpr (TOPP) {
         u4v* const rp = reinterpret_cast<u4v*>(&sh.ring[(kLRing / kLB) * tid]);
 #pragma unroll
         for (int i = 0; i < kLRing / kLB / 2; ++i) rp[i] = u4v{0u, 0u, 0u, 0u};
         if (tid < 64) sh.sub[tid] = 0ull;
         if (tid == 0) sh.nmem = 0u;
+        if constexpr (PP) {
+            u4v* const bp4 = reinterpret_cast<u4v*>(&sh.bits[(2 * kLRing / kLB) * tid]);
+#pragma unroll
+            for (int i = 0; i < 2 * kLRing / kLB / 4; ++i) bp4[i] = u4v{0u, 0u, 0u, 0u};
+            if (tid == 0) sh.np = 0u;
+        }
         lds_barrier();
     }
 #pragma unroll
@@ -172,7 +213,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
     // (i0 >= -3; indices outside the row are -inf in the stream and set no
     // bit)
     int64_t pg0 = 0, pg1 = 0;
-    const bool pen = MODE != kLongTopP && a.penalty != 1.0f && gen_range(a, row, pg0, pg1) &&
+    const bool pen = !TOPP && a.penalty != 1.0f && gen_range(a, row, pg0, pg1) &&
                      pg1 > pg0;  // (uniform)
     uint32_t* const pbm = reinterpret_cast<uint32_t*>(&sh.ring[0]);
     if (pen) {
@@ -193,6 +234,46 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
         uint32_t nb = (uint32_t)(win >> (ib & 31)) & 15u;
         if (i0 < 0) nb = (nb << (-i0)) & 15u;
         return nb;
+    };
+    // ---- PP: each distinct id is listed by the lane that sets its bit, with
+    // its value after the penalty in f64
+    int np = 0;
+    float yup = -INFINITY;   // the largest of this lane's values, rounded up
+    double ymx = -INFINITY;  //   and exactly
+    bool ybad = false;       // NaN or +inf among them
+    if constexpr (PP) {
+        if (a.penalty != 1.0f && gen_range(a, row, pg0, pg1)) {
+            for (int64_t i = pg0 + tid; i < pg1; i += kLB) {
+                const uint32_t id = a.gen_ids[i];
+                if (id >= (uint32_t)V) continue;
+                const uint32_t f = id + (uint32_t)mis, bit = 1u << (f & 31u);
+                if (atomicOr(&sh.bits[f >> 5], bit) & bit) continue;
+                const uint32_t at = atomicAdd(&sh.np, 1u);
+                if (at < (uint32_t)kLPen) {
+                    const double y = pen_value(rowp[id], penf);
+                    sh.pid[at] = id;
+                    sh.py[at] = y;
+                }
+            }
+        }
+        lds_barrier();
+        if (sh.np > (uint32_t)kLPen) return NIS_REJECT_CAPACITY;
+        np = (int)sh.np;
+        for (int j = tid; j < np; j += kLB) {
+            const double y = sh.py[j];
+            ybad |= !(y < INFINITY);
+            ymx = fmax(ymx, y);
+            yup = fmaxf(yup, pen_f32_up(y));
+        }
+    }
+    // fn(y, j): this lane's penalised values above -inf (entry j of the list)
+    auto each_pen = [&](auto&& fn) {
+        if constexpr (PP) {
+            for (int j = tid; j < np; j += kLB) {
+                const double y = sh.py[j];
+                if (y > -INFINITY) fn(y, j);
+            }
+        }
     };
 
     // =====================================================================
@@ -280,17 +361,20 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
     if ((double)chi > c64) chi = __uint_as_float(__float_as_uint(chi) - 1u);
     const float clo = (float)(c64 - (double)chi);
     const float chi64 = chi * 64.0f;
+    const double chid = (double)chi;
     float czh = chi, czl = clo;
     asm volatile("" : "+v"(czh), "+v"(czl));
 
     // ---- stream -----------------------------------------------------------
-    const float m0 = wmax_f32(r_max4(fixc(buf[0], 0)));
+    float m0 = r_max4(fixc(buf[0], 0));
+    if constexpr (PP) m0 = fmaxf(m0, yup);
+    m0 = wmax_f32(m0);
     const float Rw0 = fmaxf((m0 > -INFINITY && fabsf(m0 * chi) < 1e30f) ? ceilf(m0 * chi) : 0.0f, rfloor);
     const float tflo = (Rw0 - (float)kLSpan) * 64.0f;  // deeper elements share one bucket
     float Rz = Rw0;
     float mx = -INFINITY;  // (top-p off with a penalty: penalised values rounded up)
     double mex = -INFINITY; // top-p off with a penalty: the exact max (statistics)
-    double z = 0.0;     // the lane's mass total (2^R_z units)
+    double z = ybad ? (double)NAN : 0.0;  // the lane's mass total (2^R_z units)
     uint32_t nfin = 0;  // top-p off with stats: elements above -inf (the kept count)
     // Top-p off with a penalty: the f64 values y of a float4's penalised
     // elements give the max operand pen_f32_up(y) and the masses
@@ -351,7 +435,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
                 if (MODE == kLongAll && a.stats)
                     nfin += (uint32_t)(x.x > -INFINITY) + (uint32_t)(x.y > -INFINITY) +
                             (uint32_t)(x.z > -INFINITY) + (uint32_t)(x.w > -INFINITY);
-                if constexpr (MODE == kLongTopP) {
+                if constexpr (TOPP) {
                     const int Rs = (int)Rz + 24;
 #define NIS_LHIST(xq, eq)                                                                      \
                     {                                                                          \
@@ -376,12 +460,25 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
     } else {
         sstream(std::false_type{});
     }
+    // PP: the penalised values join the sum and the histogram
+    each_pen([&](double y, int) {
+        const float ey = (float)pen_mass(y * c64, Rz);
+        z += (double)ey;
+        const int j = d_flr(d_vmax(d_pt(y, chid) * 64.0f, tflo));
+        const uint32_t fm = (uint32_t)__builtin_amdgcn_ldexpf(ey, (int)Rz + 24 - (j >> 6));
+        __hip_atomic_fetch_add(&sh.ring[j & (kLRing - 1)], (1ull << 48) | fm, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    });
     NIS_DTS(1);
+    if constexpr (PP) {
+        mex = fmax((double)mx, ymx);
+        mx = fmaxf(mx, yup);
+    }
     mx = wmax_f32(mx);
-    if constexpr (MODE == kLongAll) {
+    if constexpr (MODE == kLongAll || PP) {
         // the wave's exact max (statistics): with a penalty, of the plain
         // logits and the penalised f64 values
-        double me = pen ? mex : (double)mx;
+        double me = (pen || PP) ? mex : (double)mx;
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) me = fmax(me, __shfl_xor(me, o));
         if (l == 0) sh.gx[w] = me;
@@ -434,9 +531,9 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
         const bool gapbad = hasd & (rr.rz - cw > 8.0f) &
                             ((R - cw < 20.0f) | ((rfloor == -INFINITY) & (rr.rz - cw > 64.0f)));
         const bool fin = (M > -INFINITY) & (M < INFINITY) & !anynan & (fabsf(M * chi) < 4096.0f) &
-                         (__ballot(gapbad) == 0ull) & (MODE != kLongTopP || (rw0hi <= R));
+                         (__ballot(gapbad) == 0ull) & (!TOPP || (rw0hi <= R));
         if (!fin) return NIS_REJECT_NONFINITE;
-        if (MODE == kLongTopP && !(R - rw0min < (float)kLSpan)) {
+        if (TOPP && !(R - rw0min < (float)kLSpan)) {
             if (rnext != nullptr && rfloor == -INFINITY) {
                 *rnext = R - (float)(kLSpan - 1);
                 return kLSpanRetry;
@@ -449,7 +546,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
     // element 0, per-element masses ev in the units of r_run), and the row's
     // result
     double Mst = (double)M;  // the row max for the statistics (top-p off: exact, f64)
-    double vfin[4] = {0.0, 0.0, 0.0, 0.0};  // top-p off: the final float4's values (penalised in f64)
+    double vfin[4] = {0.0, 0.0, 0.0, 0.0};  // top-p off, PP: the final float4's values (penalised in f64)
     auto finish = [&](const f4v& x4, uint32_t i0, const float ev[4], double r_run, double Zk,
                       double Zall, uint64_t kept) {
         int q = -1, qlast = 0;
@@ -465,7 +562,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
         }
         if (q < 0) q = qlast;
         const double u = sh.u0;
-        const double xq = (MODE == kLongAll) ? vfin[q] : (double)elem(x4, q);
+        const double xq = (MODE == kLongAll || PP) ? vfin[q] : (double)elem(x4, q);
         uint32_t tok = i0 + (uint32_t)q;
         if (u == 0.0) tok = 0u;  // r == 0 stops the reference's walk at index 0
         emit_token(a, row, tok);
@@ -632,7 +729,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
     int lv = 0, B = bp;
     unsigned long long Gc = Gp;
     uint32_t ns = nsel0, nabv = nab0;
-    float chiL = chi64;
+    float chiL = chi64, scL = 64.0f;  // (scL: chiL / c_hi)
     bool all_out = false;  // no sub-bucket passes: the whole bucket is removed
     // One refinement step of the cutoff bucket (lv, B): add(o, chiL, chiS)
     // puts its members into the 64 sub-buckets of the next level; wave 0
@@ -672,6 +769,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
         nabv = c.nab;
         if (c.rej) return false;
         chiL *= 64.0f;
+        scL *= 64.0f;
         return true;
     };
     auto sub_add = [&](float x, int o, float cl, float cs, bool valid) {
@@ -683,6 +781,13 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
                 __hip_atomic_fetch_add(&sh.sub[sb], (1ull << 48) | (unsigned long long)fm,
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
+    };
+    auto sub_pen = [&](double y, int o) {  // PP: the same for a penalised value
+        const float t = d_pt(y, chid);
+        if (d_flr(t * scL) == B)
+            __hip_atomic_fetch_add(&sh.sub[(uint32_t)d_flr(t * (scL * 64.0f)) & 63u],
+                                   (1ull << 48) | (unsigned long long)d_pfm(y * c64, o), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     // more members than the list holds: refine by reading the row again
     while (!all_out && ns > (uint32_t)kLMem) {
@@ -700,6 +805,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
                     for (int q = 0; q < 4; ++q) sub_add(elem(x, q), o, cl, cs, k < Kw);
                 }
             }
+            each_pen([&](double y, int) { sub_pen(y, o); });
         });
     }
     // ---- a second read of the row: the mass of everything above the cutoff
@@ -738,6 +844,13 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
             }
         }
     }
+    // (PP: a penalised member's entry is its place in the list, bit 31 set)
+    each_pen([&](double y, int j) {
+        if (!all_out && d_flr(d_pt(y, chid) * scL) == B) {
+            const uint32_t sm = atomicAdd(&sh.nmem, 1u);
+            if (sm < (uint32_t)kLMem) sh.lmem[sm] = LMem{0.0f, 0x80000000u | (uint32_t)j};
+        }
+    });
     const double Tabove = wsum_f64(above);
     lds_barrier();
     NIS_DTS(4);
@@ -748,7 +861,13 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
     while (!all_out && ns > (uint32_t)kDMem) {
         if (lv == kDLevels - 1) return NIS_REJECT_CAPACITY;
         all_out = !refine([&](int o, float cl, float cs) {
-            for (int j = tid; j < nm; j += kLB) sub_add(sh.lmem[j].x, o, cl, cs, true);
+            for (int j = tid; j < nm; j += kLB) {
+                const LMem m = sh.lmem[j];
+                const bool pq = PP && (m.idx >> 31);
+                sub_add(m.x, o, cl, cs, !pq);
+                if constexpr (PP)
+                    if (pq) sub_pen(sh.py[m.idx & 0x7FFFFFFFu], o);
+            }
         });
     }
     // the final bucket's members (at most kDMem) ranked exactly by wave 0
@@ -759,13 +878,30 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
         for (int j0 = 0; j0 < nm; j0 += kLB) {
             const int j = j0 + tid;
             const LMem m = sh.lmem[min(j, kLMem - 1)];
-            const bool mem = (j < nm) && (d_flr(m.x * chiL) == B);
+            float t = m.x * chiL;
+            double y = 0.0;
+            bool pq = false;
+            if constexpr (PP) {
+                pq = j < nm && (m.idx >> 31);
+                if (pq) {
+                    y = sh.py[m.idx & 0x7FFFFFFFu];
+                    t = d_pt(y, chid) * scL;
+                }
+            }
+            const bool mem = (j < nm) && (d_flr(t) == B);
             const uint64_t mb = __ballot(mem);
             if (mb) {
                 uint32_t b0 = 0u;
                 if (l == 0) b0 = atomicAdd(&sh.cnt, (uint32_t)__popcll(mb));
                 const uint32_t sm = bcast_u32(b0, 0) + lane_rank(mb);
-                if (mem) sh.mem[min(sm, (uint32_t)kDMem - 1u)] = RCand{m.x, m.idx, o, r_fm(m.x, chi, clo, o)};
+                const uint32_t sc = min(sm, (uint32_t)kDMem - 1u);
+                if (mem && !pq) sh.mem[sc] = RCand{m.x, m.idx, o, r_fm(m.x, chi, clo, o)};
+                if constexpr (PP) {
+                    if (mem && pq) {
+                        sh.mem[sc] = RCand{0.0f, m.idx, o, d_pfm(y * c64, o)};
+                        sh.my[sc] = y;
+                    }
+                }
             }
         }
     }
@@ -782,20 +918,30 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
         c.nsel = ns;
         c.rej = 0u;
         c.kcut = ~0ull;
+        c.kidx = 0u;
         c.nkept = 0u;
         if (!all_out) {
             const int n = (int)ns;
             const bool valid = l < n;
             const RCand mr = sh.mem[min(l, kDMem - 1)];
-            const unsigned long long Km = valid ? r_key(mr.x, mr.idx) : 0ull;
+            // (PP: key64 of the value, then the row index)
+            unsigned long long Km = valid ? r_key(mr.x, mr.idx) : 0ull;
+            uint32_t im = mr.idx;
+            if constexpr (PP) {
+                const bool pq = valid && (mr.idx >> 31);
+                if (pq) im = sh.pid[mr.idx & 0x7FFFFFFFu];
+                Km = valid ? key64(pq ? sh.my[min(l, kDMem - 1)] : (double)mr.x) : 0ull;
+            }
             const unsigned long long em = valid ? d_u44(mr.fm, mr.b, Ri) : 0ull;
             unsigned long long pre = 0ull;
             uint32_t rk = 0u;
             for (int j = 0; j < n; ++j) {
                 const unsigned long long Kj = rbcast_u64(Km, j);
                 const unsigned long long ej = rbcast_u64(em, j);
-                pre += (Kj > Km) ? ej : 0ull;
-                rk += (Kj > Km) ? 1u : 0u;
+                bool gt = Kj > Km;
+                if constexpr (PP) gt |= (Kj == Km) & (bcast_u32(im, j) < im);
+                pre += gt ? ej : 0ull;
+                rk += gt ? 1u : 0u;
             }
             // sampler.rs:150 in rank order
             const bool pass = valid & ((double)(Gc + pre) - (double)em <= pz);
@@ -803,6 +949,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
             if (__ballot(valid & !pass)) nkept = wmin_u32((valid && !pass) ? rk : 0xFFFFFFFFu);
             const uint64_t lastm = __ballot(valid & (rk + 1u == nkept));
             c.kcut = lastm ? rbcast_u64(Km, __ffsll((long long)lastm) - 1) : ~0ull;
+            c.kidx = lastm ? bcast_u32(im, __ffsll((long long)lastm) - 1) : 0u;
             c.nkept = nkept;
         }
         if (l == 0) sh.cut = c;
@@ -813,16 +960,44 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
     const int Bf = cut.bj;
     const unsigned long long kcut = cut.kcut;
     chiL = chi64;
-    for (int i = 0; i < cut.lv; ++i) chiL *= 64.0f;
+    scL = 64.0f;
+    for (int i = 0; i < cut.lv; ++i) {
+        chiL *= 64.0f;
+        scL *= 64.0f;
+    }
+    auto keptx = [&](float x, uint32_t idx) -> bool {
+        if constexpr (PP) {
+            const int F = d_flr(x * chiL);
+            return (F > Bf) | ((F == Bf) && d_pkeep(key64((double)x), idx, kcut, cut.kidx));
+        } else {
+            return d_kept(x, idx, chiL, Bf, kcut);
+        }
+    };
+    auto kepty = [&](double y, uint32_t idx) -> bool {  // PP: a penalised value
+        const int F = d_flr(d_pt(y, chid) * scL);
+        return (F > Bf) | ((F == Bf) && d_pkeep(key64(y), idx, kcut, cut.kidx));
+    };
     // the listed members that are kept join their wave's kept mass
     const int span = 4 * 64 * cpw;  // row indices per wave
     for (int j = tid; j < nm; j += kLB) {
         const LMem m = sh.lmem[j];
-        if (d_kept(m.x, m.idx, chiL, Bf, kcut)) {
+        if (PP && (m.idx >> 31)) continue;
+        if (keptx(m.x, m.idx)) {
             const int ow = min((int)((m.idx + (uint32_t)mis) / (uint32_t)span), kLW - 1);
             __hip_atomic_fetch_add(&sh.tmem[ow], (double)r_mass(m.x, czh, czl, sh.rec[ow].rz),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
+    }
+    // (PP: so do the kept penalised values)
+    if constexpr (PP) {
+        each_pen([&](double y, int j) {
+            const uint32_t idx = sh.pid[j];
+            if (kepty(y, idx)) {
+                const int ow = min((int)((idx + (uint32_t)mis) / (uint32_t)span), kLW - 1);
+                __hip_atomic_fetch_add(&sh.tmem[ow], (double)(float)pen_mass(y * c64, sh.rec[ow].rz),
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+        });
     }
     lds_barrier();
     if (l == 0) sh.tw[w] = ldexp(Tabove + sh.tmem[w], (int)(Rz - R));  // 2^R units (exact)
@@ -854,14 +1029,21 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
 #pragma unroll
         for (int i = 0; i < kLD; ++i) {
             const int k = k0 + i;
-            const f4v x = fixc(buf[i], k);
+            const f4v x = fixr(buf[i], k);
             buf[i] = ld(k + kLD);
             if (k < Kw && kc < 0) {
                 float ev[4];
+                const uint32_t nb = ppnib(k);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const float xq = elem(x, q);
-                    ev[q] = d_kept(xq, (uint32_t)(NIS_LIDX(k) + q), chiL, Bf, kcut) ? r_mass(xq, czh, czl, Rz) : 0.0f;
+                    const uint32_t idx = (uint32_t)(NIS_LIDX(k) + q);
+                    if (PP && ((nb >> q) & 1u)) {
+                        const double y = pen_value(xq, penf);
+                        ev[q] = kepty(y, idx) ? (float)pen_mass(y * c64, Rz) : 0.0f;
+                    } else {
+                        ev[q] = keptx(xq, idx) ? r_mass(xq, czh, czl, Rz) : 0.0f;
+                    }
                 }
                 const float v = (ev[0] + ev[1]) + (ev[2] + ev[3]);
                 const double ct = wsum_f64((double)v);
@@ -893,6 +1075,16 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row, Lon
         rkc = rklast;
 #pragma unroll
         for (int q = 0; q < 4; ++q) evc[q] = evl[q];
+    }
+    if constexpr (PP) {
+        const uint32_t nb = ppnib(kc);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            vfin[q] = ((nb >> q) & 1u) ? pen_value(elem(xc, q), penf) : (double)elem(xc, q);
+        double me = rv ? sh.gx[l] : -INFINITY;
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) me = fmax(me, __shfl_xor(me, o));
+        Mst = me;
     }
     NIS_DTS(8);
     {
@@ -929,6 +1121,31 @@ __global__ __launch_bounds__(kLB, 2) void sample_rows_long_kernel(RowArgs a) {
         if (reject == NIS_REJECT_NONE) return;
         // (|R| < 4096: the retry's floor fits the token's low 14 bits)
         if (reject == kLSpanRetry) reject = kLSpanFlag | ((uint32_t)((int)rn + 8192) & 0x3FFFu);
+    }
+    if (threadIdx.x == 0) a.tokens[row] = kLPending | reject;
+}
+
+// Long top-p rows with a repetition-penalty history (V <= kLPenMaxV, at most
+// kLPen distinct ids).  The three reads of the row (one from HBM, two from the
+// MALL or L2) and an LDS atomic an element bound it; the penalised elements are
+// masked out of each read by a bitmap and join as f64 values from a short list.
+// A row whose span asks for it runs once more with raised references.
+// A decode step of 128 rows of V = 128256, top-p 0.9, penalty 1.1, 256-id
+// histories: 1092 us on the general path (radix passes over f64 keys), 104 here.
+__global__ __launch_bounds__(kLB) void sample_rows_long_pen_kernel(RowArgs a) {
+    __shared__ LongPenShared sh;
+    const int row = (int)blockIdx.x;
+    if (a.done != nullptr && a.done[row]) return;  // a finished sequence (decode step)
+    uint32_t reject = NIS_REJECT_SHAPE;
+    if (long_eligible<kLongTopPPen>(a, row)) {
+        float rfl = -INFINITY, rn = 0.0f;
+        for (;;) {
+            reject = long_row<kLongTopPPen>(a, row, sh, NIS_REJECT_NONE, rfl, &rn);
+            if (reject != kLSpanRetry) break;  // (returned at rfl = -inf only)
+            rfl = rn;
+            __syncthreads();
+        }
+        if (reject == NIS_REJECT_NONE) return;
     }
     if (threadIdx.x == 0) a.tokens[row] = kLPending | reject;
 }
