@@ -175,7 +175,7 @@ nis::RowArgs row_args(const float* d_logits, int64_t ld, int64_t V, const nis_pa
 //   - 0 < top-k < V with a penalty history, or with V > 53245 (to 262141), at
 //     any top-p > 0: the 1024-lane top-k path (only the row's head is kept);
 //   - 53245 < V <= 262080, 0 < top-p < 1, no top-k, with a penalty history: the
-//     512-lane long-row kernel's penalty form, then the general path on the
+//     1024-lane long-row kernel's penalty form, then the general path on the
 //     rows it declined;
 //   - anything else (V < 256, top-p <= 0, top-k past 262141, a penalty history
 //     on rows of V > 262080): the 512-lane general kernel.
@@ -249,7 +249,7 @@ int launch_rows(nis_ctx* ctx, const nis::RowArgs& a, int32_t B) {
                a.top_p > 0.0f && a.top_p < 1.0f) {
         // long top-p rows with a penalty history, then the rows it declined
         // (non-finite, more than kLPen distinct ids, exact-tie overflow)
-        hipLaunchKernelGGL(nis::sample_rows_long_pen_kernel, dim3((unsigned)B), dim3(nis::kLB), 0, ctx->stream, a);
+        hipLaunchKernelGGL(nis::sample_rows_long_pen_kernel, dim3((unsigned)B), dim3(nis::kLPB), 0, ctx->stream, a);
         hipLaunchKernelGGL(nis::sample_rows_pending_kernel, dim3((unsigned)std::min(B, 256)),
                            dim3(nis::kBlock), 0, ctx->stream, a, B);
     } else if (nis::topk_eligible(a)) {

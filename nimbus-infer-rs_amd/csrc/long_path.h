@@ -38,11 +38,11 @@
 namespace nis {
 
 constexpr int kLB = 512;              // lanes per workgroup (two workgroups share a CU)
-constexpr int kLW = kLB / 64;         // waves per workgroup
 constexpr int kLD = 4;                // loads in flight per lane
 constexpr int kLRing = 4096;          // histogram ring: 64 octaves of 64 buckets
 constexpr int kLSpan = 32;            // octaves searched below R (and folded below R_w0)
-constexpr int kLQ = 64 * kLSpan / kLB;  // searched buckets per lane
+constexpr int kLPB = 1024;            // lanes with a top-p penalty history (LDS holds one workgroup per CU)
+constexpr int kLWMax = kLPB / 64;
 constexpr uint32_t kLPending = 0xFFF00000u;  // token of a declined row (| reject code)
 constexpr int kLMem = 2048;           // members of the cutoff bucket listed by the second read
 
@@ -61,16 +61,16 @@ struct LongShared {
     LMem lmem[kLMem];                 // the cutoff bucket's members (second read)
     RCand mem[kDMem];                 // members of the final bucket
     unsigned long long sub[64];       // refinement histogram of the cutoff bucket
-    DRec rec[kLW];
-    unsigned long long wtm[kLW];      // search: each wave's bucket mass
-    unsigned long long wlo[kLW];      //   and that of the 32 octaves below the search
-    uint32_t wtc[kLW];                //   and count
-    DCand cand[kLW];
-    double tw[kLW];                   // per-wave kept mass (2^R units)
-    double tmem[kLW];                 // per-wave kept mass of listed members (2^R_z units)
-    uint32_t nfin[kLW];               // top-p off: each wave's elements above -inf (stats)
-    double gx[kLW];                   // greedy: each wave's max (penalised values in f64)
-    int32_t gi[kLW];                  //   and the first index holding it
+    DRec rec[kLWMax];
+    unsigned long long wtm[kLWMax];      // search: each wave's bucket mass
+    unsigned long long wlo[kLWMax];      //   and that of the 32 octaves below the search
+    uint32_t wtc[kLWMax];                //   and count
+    DCand cand[kLWMax];
+    double tw[kLWMax];                   // per-wave kept mass (2^R units)
+    double tmem[kLWMax];                 // per-wave kept mass of listed members (2^R_z units)
+    uint32_t nfin[kLWMax];               // top-p off: each wave's elements above -inf (stats)
+    double gx[kLWMax];                   // greedy: each wave's max (penalised values in f64)
+    int32_t gi[kLWMax];                  //   and the first index holding it
     DCut cut;
     double u0;                        // the draw
     uint32_t nmem;                    // members listed by the second read
@@ -123,6 +123,8 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
                                              uint32_t prior = NIS_REJECT_NONE, const float rfloor = -INFINITY,
                                              float* const rnext = nullptr) {
     constexpr bool PP = MODE == kLongTopPPen, TOPP = MODE == kLongTopP || PP;
+    constexpr int LB = PP ? kLPB : kLB, LW = LB / 64;
+    constexpr int LQ = 64 * kLSpan / LB;  // searched buckets per lane
     const int l = lane_id();
     const int w = __builtin_amdgcn_readfirstlane(wave_id());
     const int tid = (int)threadIdx.x;
@@ -133,7 +135,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     const int f_lo = mis ? 1 : 0;          // first float4 slot lying fully inside the row
     const int f_hi = (V + mis - 4) >> 2;   // last one
     const int nsl = (V + mis + 3) >> 2;    // slots touching the row
-    const int cpw = (((nsl + 63) >> 6) + kLW - 1) / kLW;  // chunks per wave
+    const int cpw = (((nsl + 63) >> 6) + LW - 1) / LW;  // chunks per wave
     const int wbase = 64 * cpw * w;
     const int Kw = min(max((nsl - wbase + 63) >> 6, 0), cpw);
     const int slot0 = wbase + l;
@@ -185,15 +187,15 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     buf[0] = ld(0);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (TOPP) {
-        u4v* const rp = reinterpret_cast<u4v*>(&sh.ring[(kLRing / kLB) * tid]);
+        u4v* const rp = reinterpret_cast<u4v*>(&sh.ring[(kLRing / LB) * tid]);
 #pragma unroll
-        for (int i = 0; i < kLRing / kLB / 2; ++i) rp[i] = u4v{0u, 0u, 0u, 0u};
+        for (int i = 0; i < kLRing / LB / 2; ++i) rp[i] = u4v{0u, 0u, 0u, 0u};
         if (tid < 64) sh.sub[tid] = 0ull;
         if (tid == 0) sh.nmem = 0u;
         if constexpr (PP) {
-            u4v* const bp4 = reinterpret_cast<u4v*>(&sh.bits[(2 * kLRing / kLB) * tid]);
+            u4v* const bp4 = reinterpret_cast<u4v*>(&sh.bits[(2 * kLRing / LB) * tid]);
 #pragma unroll
-            for (int i = 0; i < 2 * kLRing / kLB / 4; ++i) bp4[i] = u4v{0u, 0u, 0u, 0u};
+            for (int i = 0; i < 2 * kLRing / LB / 4; ++i) bp4[i] = u4v{0u, 0u, 0u, 0u};
             if (tid == 0) sh.np = 0u;
         }
         lds_barrier();
@@ -218,9 +220,9 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     uint32_t* const pbm = reinterpret_cast<uint32_t*>(&sh.ring[0]);
     if (pen) {
         const int nwd = ((int)a.V + 31) / 32 + 1;  // (+1: the window's second word)
-        for (int i = tid; i < nwd; i += kLB) pbm[i] = 0u;
+        for (int i = tid; i < nwd; i += LB) pbm[i] = 0u;
         lds_barrier();
-        for (int64_t i = pg0 + tid; i < pg1; i += kLB) {
+        for (int64_t i = pg0 + tid; i < pg1; i += LB) {
             const uint32_t id = a.gen_ids[i];
             if (id < (uint32_t)a.V) atomicOr(&pbm[id >> 5], 1u << (id & 31));
         }
@@ -243,7 +245,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     bool ybad = false;       // NaN or +inf among them
     if constexpr (PP) {
         if (a.penalty != 1.0f && gen_range(a, row, pg0, pg1)) {
-            for (int64_t i = pg0 + tid; i < pg1; i += kLB) {
+            for (int64_t i = pg0 + tid; i < pg1; i += LB) {
                 const uint32_t id = a.gen_ids[i];
                 if (id >= (uint32_t)V) continue;
                 const uint32_t f = id + (uint32_t)mis, bit = 1u << (f & 31u);
@@ -259,7 +261,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
         lds_barrier();
         if (sh.np > (uint32_t)kLPen) return NIS_REJECT_CAPACITY;
         np = (int)sh.np;
-        for (int j = tid; j < np; j += kLB) {
+        for (int j = tid; j < np; j += LB) {
             const double y = sh.py[j];
             ybad |= !(y < INFINITY);
             ymx = fmax(ymx, y);
@@ -269,7 +271,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     // fn(y, j): this lane's penalised values above -inf (entry j of the list)
     auto each_pen = [&](auto&& fn) {
         if constexpr (PP) {
-            for (int j = tid; j < np; j += kLB) {
+            for (int j = tid; j < np; j += LB) {
                 const double y = sh.py[j];
                 if (y > -INFINITY) fn(y, j);
             }
@@ -341,7 +343,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
             sh.gi[w] = bad ? -1 : wi;
         }
         lds_barrier();
-        const bool rv = l < kLW;
+        const bool rv = l < LW;
         const double gx = rv ? sh.gx[l] : -INFINITY;
         const int gi = rv ? sh.gi[l] : 0x7FFFFFFF;
         if (__ballot(rv & (gi < 0))) return NIS_REJECT_NONFINITE;
@@ -488,7 +490,8 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
         const double zw = wsum_f64(z);
         const uint32_t nf = (MODE == kLongAll && a.stats) ? wsum_u32(nfin) : 0u;
         if (l == 0) {
-            sh.rec[w] = DRec{mx, Rz, Rw0, nan_seen | (Kw > 0 ? 2u : 0u)};
+            // (PP: a wave past the row may hold penalised values)
+            sh.rec[w] = DRec{mx, Rz, Rw0, nan_seen | ((Kw > 0 || (PP && mx > -INFINITY)) ? 2u : 0u)};
             sh.tw[w] = zw;  // top-p off: the wave's total (2^R_z units)
             sh.nfin[w] = nf;
         }
@@ -506,7 +509,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     // ---- B1 ---------------------------------------------------------------------
     lds_barrier();
     NIS_DTS(2);
-    const bool rv = l < kLW;
+    const bool rv = l < LW;
     const DRec rr = sh.rec[rv ? l : 0];
     const bool has = rv && (rr.flags & 2u);
     const float M = wmax_f32(has ? rr.mx : -INFINITY);
@@ -641,7 +644,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
         const uint64_t hl = __ballot((sl > 0.0) & (lincl >= rk));
         const uint64_t nzl = __ballot(sl > 0.0);
         const int lc = hl ? (__ffsll((long long)hl) - 1) : (63 - __clzll((long long)(nzl | 1ull)));
-        const uint32_t nkept = a.stats ? wsum_u32(l < kLW ? sh.nfin[l] : 0u) : 0u;
+        const uint32_t nkept = a.stats ? wsum_u32(l < LW ? sh.nfin[l] : 0u) : 0u;
         if (l == lc) finish(xc, (uint32_t)NIS_LIDX(kc), ev, rk - (lincl - sl), Z, 0.0, (uint64_t)nkept);
         return NIS_REJECT_NONE;
     }
@@ -649,11 +652,11 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     // =====================================================================
     // ---- top-p: cutoff search over the 32 octaves below R ----------------
     const float p = a.top_p;
-    const int jt0 = 64 * Ri - 64 * kLQ * w - kLQ * l;  // lane: buckets jt0 .. jt0 - kLQ + 1
-    unsigned long long bm[kLQ];
-    uint32_t bc[kLQ];
+    const int jt0 = 64 * Ri - 64 * LQ * w - LQ * l;  // lane: buckets jt0 .. jt0 - LQ + 1
+    unsigned long long bm[LQ];
+    uint32_t bc[LQ];
 #pragma unroll
-    for (int q = 0; q < kLQ; ++q) {
+    for (int q = 0; q < LQ; ++q) {
         const int j = jt0 - q;
         const unsigned long long v = sh.ring[j & (kLRing - 1)];
         bc[q] = (uint32_t)(v >> 48);
@@ -662,7 +665,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     unsigned long long lm = 0ull;
     uint32_t lcn = 0u;
 #pragma unroll
-    for (int q = 0; q < kLQ; ++q) {
+    for (int q = 0; q < LQ; ++q) {
         lm += bm[q];
         lcn += bc[q];
     }
@@ -671,7 +674,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     // the 32 octaves below the search (and the folded bucket) still count in Z
     unsigned long long lo = 0ull;
 #pragma unroll
-    for (int q = 0; q < kLQ; ++q) {
+    for (int q = 0; q < LQ; ++q) {
         const int j = jt0 - q - 64 * kLSpan;
         lo += d_u44(sh.ring[j & (kLRing - 1)], j >> 6, Ri);
     }
@@ -686,7 +689,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     const uint32_t wci = rscan_u32(rv ? sh.wtc[l] : 0u);
     const unsigned long long wli = rscan16_u64(rv ? sh.wlo[l] : 0ull);
     // Z in 2^(R - 44) units
-    const unsigned long long Z = rbcast_u64(wmi, kLW - 1) + rbcast_u64(wli, kLW - 1);
+    const unsigned long long Z = rbcast_u64(wmi, LW - 1) + rbcast_u64(wli, LW - 1);
     const double pz = (double)p * (double)Z;
     {
         unsigned long long G = (w > 0 ? rbcast_u64(wmi, w - 1) : 0ull) + (im - lm);
@@ -695,7 +698,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
         unsigned long long gp_ = 0ull;
         uint32_t np_ = 0u, cp_ = 0u;
 #pragma unroll
-        for (int q = 0; q < kLQ; ++q) {
+        for (int q = 0; q < LQ; ++q) {
             const int j = jt0 - q;
             if ((bc[q] != 0u) && ((double)G - d_mup(j, 0, Ri) <= pz)) {
                 jp = j;
@@ -861,7 +864,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     while (!all_out && ns > (uint32_t)kDMem) {
         if (lv == kDLevels - 1) return NIS_REJECT_CAPACITY;
         all_out = !refine([&](int o, float cl, float cs) {
-            for (int j = tid; j < nm; j += kLB) {
+            for (int j = tid; j < nm; j += LB) {
                 const LMem m = sh.lmem[j];
                 const bool pq = PP && (m.idx >> 31);
                 sub_add(m.x, o, cl, cs, !pq);
@@ -875,7 +878,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     lds_barrier();
     if (!all_out && ns > 0u) {
         const int o = B >> (6 * (lv + 1));
-        for (int j0 = 0; j0 < nm; j0 += kLB) {
+        for (int j0 = 0; j0 < nm; j0 += LB) {
             const int j = j0 + tid;
             const LMem m = sh.lmem[min(j, kLMem - 1)];
             float t = m.x * chiL;
@@ -905,7 +908,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
             }
         }
     }
-    if (tid < kLW) sh.tmem[tid] = 0.0;
+    if (tid < LW) sh.tmem[tid] = 0.0;
     lds_barrier();
     NIS_DTS(5);
     if (!all_out && sh.cnt != ns) return NIS_REJECT_BUCKET;
@@ -979,11 +982,11 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
     };
     // the listed members that are kept join their wave's kept mass
     const int span = 4 * 64 * cpw;  // row indices per wave
-    for (int j = tid; j < nm; j += kLB) {
+    for (int j = tid; j < nm; j += LB) {
         const LMem m = sh.lmem[j];
         if (PP && (m.idx >> 31)) continue;
         if (keptx(m.x, m.idx)) {
-            const int ow = min((int)((m.idx + (uint32_t)mis) / (uint32_t)span), kLW - 1);
+            const int ow = min((int)((m.idx + (uint32_t)mis) / (uint32_t)span), LW - 1);
             __hip_atomic_fetch_add(&sh.tmem[ow], (double)r_mass(m.x, czh, czl, sh.rec[ow].rz),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
@@ -993,7 +996,7 @@ __device__ __forceinline__ uint32_t long_row(const RowArgs a, const int row,
         each_pen([&](double y, int j) {
             const uint32_t idx = sh.pid[j];
             if (kepty(y, idx)) {
-                const int ow = min((int)((idx + (uint32_t)mis) / (uint32_t)span), kLW - 1);
+                const int ow = min((int)((idx + (uint32_t)mis) / (uint32_t)span), LW - 1);
                 __hip_atomic_fetch_add(&sh.tmem[ow], (double)(float)pen_mass(y * c64, sh.rec[ow].rz),
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
@@ -1131,8 +1134,9 @@ __global__ __launch_bounds__(kLB, 2) void sample_rows_long_kernel(RowArgs a) {
 // masked out of each read by a bitmap and join as f64 values from a short list.
 // A row whose span asks for it runs once more with raised references.
 // A decode step of 128 rows of V = 128256, top-p 0.9, penalty 1.1, 256-id
-// histories: 1092 us on the general path (radix passes over f64 keys), 104 here.
-__global__ __launch_bounds__(kLB) void sample_rows_long_pen_kernel(RowArgs a) {
+// histories: 1092 us on the general path (radix passes over f64 keys), 92 here
+// (104 with 512 lanes: LDS holds one workgroup per CU either way).
+__global__ __launch_bounds__(kLPB) void sample_rows_long_pen_kernel(RowArgs a) {
     __shared__ LongPenShared sh;
     const int row = (int)blockIdx.x;
     if (a.done != nullptr && a.done[row]) return;  // a finished sequence (decode step)
