@@ -400,7 +400,16 @@ __global__ __launch_bounds__(256) void lm_head_row_kernel(LmHeadArgs a, int log2
 
     constexpr int D = LhRowCfg<FMT>::D;
     RunT ring[D][KM];
-    auto load_step = [&](int it, RunT* dst) {
+    // GROUPED: the runs' scales travel with them in the ring.  Loaded where they
+    // were used, each step waited for memory: 4096 x 128256 in groups of 128,
+    // int4 109 -> 74 us (67 without groups), int8 126 -> 101.  (16 steps a wave
+    // instead of 4, which read the hidden row a quarter as often, were slower:
+    // int4 94, without groups 90.)
+    float rsc[D][KM];
+    int gid[KM];  // the runs' groups
+#pragma unroll
+    for (int k = 0; k < KM; ++k) gid[k] = GROUPED ? lh_group_of(a, min(li + k * L, runs - 1) * R) : 0;
+    auto load_step = [&](int it, RunT* dst, float* sdst) {
         const int64_t vl = min(wave_row0 + it * P + gl, a.V - 1);
         const uint8_t* wrow = (const uint8_t*)a.w + vl * row_bytes;
 #pragma unroll
@@ -411,10 +420,11 @@ __global__ __launch_bounds__(256) void lm_head_row_kernel(LmHeadArgs a, int log2
             const RunT v = *(const RunT*)(wrow + (int64_t)min(j, runs - 1) * RB);
             RunT z{};
             dst[k] = j < runs ? v : z;
+            if (GROUPED) sdst[k] = a.scales[vl * a.groups + gid[k]];
         }
     };
 #pragma unroll
-    for (int it = 0; it < D; ++it) load_step(it, ring[it]);
+    for (int it = 0; it < D; ++it) load_step(it, ring[it], rsc[it]);
     float xr[KM][R];
     float sx[KM];
 #pragma unroll
@@ -435,18 +445,21 @@ __global__ __launch_bounds__(256) void lm_head_row_kernel(LmHeadArgs a, int log2
 #pragma unroll
     for (int it = 0; it < ITER; ++it) {
         const int64_t v = wave_row0 + it * P + gl;
-        const int64_t vl = min(v, a.V - 1);
         RunT cur[KM];
+        float sc[KM];
 #pragma unroll
-        for (int k = 0; k < KM; ++k) cur[k] = ring[it % D][k];
-        if (it + D < ITER) load_step(it + D, ring[it % D]);
+        for (int k = 0; k < KM; ++k) {
+            cur[k] = ring[it % D][k];
+            if (GROUPED) sc[k] = rsc[it % D][k];
+        }
+        if (it + D < ITER) load_step(it + D, ring[it % D], rsc[it % D]);
         float acc = 0.f;
 #pragma unroll
         for (int k = 0; k < KM; ++k) {
             const int j = li + k * L;
             if (j < runs) {
                 const float part = lh_run_dot<FMT>(cur[k], xr[k], sx[k]);
-                if (GROUPED) acc = fmaf(part, a.scales[vl * a.groups + lh_group_of(a, j * R)], acc);
+                if (GROUPED) acc = fmaf(part, sc[k], acc);
                 else acc += part;
             }
         }
